@@ -50,6 +50,7 @@ struct as_ctx {
   float* d_zero = nullptr;  // 1,024 zeros the scan's idle loads read
   as_launch::LpPart* d_lp = nullptr;  // log-probabilities: per row, its parts' sums and lists
   uint64_t* d_mv_partials = nullptr;  // head_argmax: each matvec workgroup's best key
+  uint64_t* d_arg = nullptr;  // argmax_rows: each slice's best key, then the rows' counts of ended slices
   as_launch::RowOrder order{};  // the scan's row order for the current call
   std::vector<std::pair<double, uint32_t>> order_cost;  // its sort keys (kept: no allocation per call)
   std::vector<RowParams> rows;  // the call's parameter blocks as built on the host (max_rows, kept)
@@ -412,6 +413,7 @@ int as_destroy(as_ctx* c) {
   (void)hipFree(c->d_zero);
   (void)hipFree(c->d_lp);
   (void)hipFree(c->d_mv_partials);
+  (void)hipFree(c->d_arg);
   for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
   for (int b = 0; b < 2; ++b)
     if (c->h_block[b]) (void)hipHostFree(c->h_block[b]);
@@ -466,6 +468,9 @@ int as_create(int device, void* hip_stream, uint32_t max_rows, uint32_t max_voca
   if (e == hipSuccess) e = hipMalloc(&c->d_scratch, sizeof(uint32_t) * (uint64_t)max_rows * c->scratch_stride);
   if (e == hipSuccess) e = hipMalloc(&c->d_vstatus, sizeof(uint32_t) * max_rows);
   if (e == hipSuccess) e = hipMalloc(&c->d_mv_partials, sizeof(uint64_t) * as_launch::kMatvecGroups);
+  const size_t arg_best = sizeof(uint64_t) * 2 * as_launch::kArgGroups, arg_arrived = sizeof(uint32_t) * as_launch::kArgGroups;
+  if (e == hipSuccess) e = hipMalloc(&c->d_arg, arg_best + arg_arrived);
+  if (e == hipSuccess) e = hipMemset(c->d_arg, 0, arg_best + arg_arrived);
   if (e == hipSuccess)
     e = hipMalloc(&c->d_lp, sizeof(as_launch::LpPart) * as_launch::lp_capacity(max_rows, max_vocab));
   if (e == hipSuccess) e = hipMalloc(&c->d_zero, sizeof(float) * 1024);
@@ -572,8 +577,9 @@ int as_argmax_rows(as_ctx* c, const float* logits, uint64_t row_stride, uint32_t
     return fail(c, AS_ERR_INVALID, "as_argmax_rows: bad pointers or row_stride < n");
   AS_HIP(c, hipSetDevice(c->device));
   const bool vec = aligned16(logits) && (row_stride % 4 == 0);
-  AS_HIP(c, as_launch::argmax_rows(c->stream, vec, logits, row_stride, n, n_rows, ids, rows_out,
-                                   embd, row_bytes, slot));
+  uint32_t* arrived = reinterpret_cast<uint32_t*>(c->d_arg + 2 * as_launch::kArgGroups);
+  AS_HIP(c, as_launch::argmax_rows(c->stream, vec, logits, row_stride, n, n_rows, c->d_arg, arrived, ids,
+                                   rows_out, embd, row_bytes, slot));
   return AS_OK;
 }
 
