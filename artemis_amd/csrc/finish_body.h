@@ -48,6 +48,10 @@ struct Shared {
   // whether the kept set runs past them, and the bounds on u.
   uint32_t fp_m, fp_past;
   uint32_t vast;  // a slice found min-p's floor set vast
+  double ex_total;     // the reference's total of the row in index order, when ex_have
+  uint32_t ex_have;
+  double fold_sum[2];  // exact_fold: the running sum after a tile, and where it passed its limit
+  uint32_t fold_hit[2];
   // The row's parameters, RNG state and history bounds, loaded with the list of flagged rows at the
   // kernel's start (row_prefetch), so that a row that first takes parts of S finds them in LDS.
   RowParams prm;
@@ -77,25 +81,95 @@ __device__ double block_exclusive_scan_f64(double x, double* wave_tot) {
 
 // --- the exact-order path ---------------------------------------------------------------------
 
-// Thread 0's left-to-right f64 fold of term(i), i in [0, m), staged through LDS in tiles that all
-// threads fill. Returns the sum to every thread.
-template <class Term>
-__device__ __forceinline__ double seq_fold(Shared& sh, uint32_t m, Term term) {
-  double* stage = sh.wd;
-  double acc = 0.0;
-  for (uint32_t t0 = 0; t0 < m; t0 += kStage) {
-    const uint32_t c = min((uint32_t)kStage, m - t0);
-    for (uint32_t i = threadIdx.x; i < c; i += kThreads) stage[i] = term(t0 + i);
-    __syncthreads();
-    if (threadIdx.x == 0)
-      for (uint32_t i = 0; i < c; ++i) acc = __dadd_rn(acc, stage[i]);
-    __syncthreads();
+// The reference's left-to-right f64 folds of positive terms, rounding for rounding, by a block. While the
+// running sum s stays in one binade [2^e, 2^(e+1)), every addition rounds to the grid of U = 2^(e-52), and s
+// lies on that grid: s + w rounds to s plus w rounded to the grid, except that a w halfway between two grid
+// points rounds to the even sum, which depends on s. So 256 terms at a time, wave 0 rounds each to the grid
+// ((w + 2^e) - 2^e, exact for w < 2^e) and adds the results (multiples of U under 2^(e+1): exact in any
+// order); only where a term lies halfway, or the sum leaves the binade or passes `limit`, does it add them
+// one by one. (A uniformly spread fold has about one halfway term per binade.)
+//
+// fold_tile: wave 0 folds w[0 .. c) (LDS) onto s, until the running sum passes limit (ge: reaches it);
+// *hit is then the index of the term that did (else kNone).
+__device__ __noinline__ double fold_tile(const double* w, uint32_t c, double s, double limit, bool ge, uint32_t* hit) {
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  constexpr uint32_t kPer = 4;
+  *hit = kNone;
+  for (uint32_t b = 0; b < c; b += kPer * kWave) {
+    double x[kPer];
+#pragma unroll
+    for (uint32_t q = 0; q < kPer; ++q) {
+      const uint32_t i = b + q * kWave + lane;
+      x[q] = i < c ? w[i] : 0.0;
+    }
+    if (s > 0x1p-900) {
+      const double one = __longlong_as_double(__double_as_longlong(s) & 0x7FF0000000000000ll);  // 2^e
+      const double half = one * 0x1p-53;                                                       // U / 2
+      bool off = false;
+      double r = 0.0;
+#pragma unroll
+      for (uint32_t q = 0; q < kPer; ++q) {
+        const double g = __dsub_rn(__dadd_rn(x[q], one), one);
+        off = off || !(x[q] < one) || fabs(__dsub_rn(x[q], g)) == half;
+        r = __dadd_rn(r, g);
+      }
+      const double s2 = __dadd_rn(s, wave_sum_f64(r));
+      if (__ballot(off) == 0ull && s2 < 2.0 * one && !(ge ? s2 >= limit : s2 > limit)) {
+        s = s2;
+        continue;
+      }
+    }
+    for (uint32_t q = 0; q < kPer && b + q * kWave < c; ++q) {
+      const double cum = wave_seq_prefix(q == 0 ? x[0] : q == 1 ? x[1] : q == 2 ? x[2] : x[3], s);
+      const uint32_t i = b + q * kWave + lane;
+      const uint64_t m = __ballot(i < c && (ge ? cum >= limit : cum > limit));
+      if (m) {
+        *hit = b + q * kWave + (uint32_t)__builtin_ctzll(m);
+        return s;
+      }
+      s = wave_lane63(cum);
+    }
   }
-  if (threadIdx.x == 0) sh.sum = acc;
+  return s;
+}
+
+// The fold of term(i), i in [0, m): wave 0 folds a tile in LDS (sh.wd) while the others fill the next. Returns
+// the sum to every thread, or, once the running sum passes limit (ge: reaches it), with *first the index of
+// the term that did (kNone: none).
+template <class Term>
+__device__ __forceinline__ double exact_fold(Shared& sh, uint32_t m, double limit, bool ge, uint32_t* first, Term term) {
+  static_assert(2 * kStage <= kCap, "two tiles");
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t i = tid; i < min((uint32_t)kStage, m); i += kThreads) sh.wd[i] = term(i);
   __syncthreads();
-  const double r = sh.sum;
+  double s = 0.0;
+  uint32_t hit = kNone;
+  for (uint32_t t = 0, t0 = 0; t0 < m; ++t, t0 += kStage) {
+    if (tid < kWave) {
+      uint32_t h;
+      s = fold_tile(sh.wd + (t & 1u) * kStage, min((uint32_t)kStage, m - t0), s, limit, ge, &h);
+      if (tid == 0) {
+        sh.fold_sum[t & 1u] = s;
+        sh.fold_hit[t & 1u] = h == kNone ? kNone : t0 + h;
+      }
+    } else {
+      const uint32_t n0 = t0 + kStage;
+      for (uint32_t i = tid - kWave; n0 < m && i < min((uint32_t)kStage, m - n0); i += kThreads - kWave)
+        sh.wd[((t + 1) & 1u) * kStage + i] = term(n0 + i);
+    }
+    __syncthreads();
+    s = sh.fold_sum[t & 1u];
+    hit = sh.fold_hit[t & 1u];
+    if (hit != kNone) break;
+  }
   __syncthreads();
-  return r;
+  *first = hit;
+  return s;
+}
+template <class Term>
+__device__ __forceinline__ double exact_sum(Shared& sh, uint32_t m, Term term) {
+  uint32_t first;
+  return exact_fold(sh, m, __builtin_inf(), false, &first, term);
 }
 
 // One stable pass of an LSD radix sort on 8 bits: (src_key, src_id) -> (dst_key, dst_id).
@@ -217,31 +291,10 @@ __device__ __noinline__ void exact_row(const FinishArgs& a, const RowParams& p, 
     const uint32_t k = p.top_k;
     keep = k;
     if (p.top_p < 1.0f) {
-      const double total = seq_fold(sh, k, [&](uint32_t j) { return w_one(rv(j)); });
-      // The cumulative walk, thread 0 over staged weights.
-      if (tid == 0) sh.done = 0;
-      for (uint32_t t0 = 0; t0 < k; t0 += kStage) {
-        const uint32_t c = min((uint32_t)kStage, k - t0);
-        for (uint32_t i = tid; i < c; i += kThreads) sh.wd[i] = w_one(rv(t0 + i));
-        __syncthreads();
-        if (tid == 0) {
-          double cum = sh.sum;  // carried between tiles
-          if (t0 == 0) cum = 0.0;
-          for (uint32_t i = 0; i < c; ++i) {
-            cum = __dadd_rn(cum, __ddiv_rn(sh.wd[i], total));
-            if (cum >= top_p) {
-              sh.keep = t0 + i + 1;
-              sh.done = 1;
-              break;
-            }
-          }
-          sh.sum = cum;
-        }
-        __syncthreads();
-        if (sh.done) break;
-      }
-      if (sh.done) keep = sh.keep;
-      __syncthreads();
+      const double total = exact_sum(sh, k, [&](uint32_t j) { return w_one(rv(j)); });
+      uint32_t first;
+      exact_fold(sh, k, top_p, true, &first, [&](uint32_t j) { return __ddiv_rn(w_one(rv(j)), total); });
+      if (first != kNone) keep = first + 1;
     }
     if (has_floor) {
       uint32_t first = keep;
@@ -250,46 +303,23 @@ __device__ __noinline__ void exact_row(const FinishArgs& a, const RowParams& p, 
       keep = block_min_u32<kWaves>(first, sh.red_u);
     }
   } else if (p.top_p < 1.0f || has_floor) {
-    double total1 = 0.0;
-    if (p.top_p < 1.0f) total1 = seq_fold(sh, n, [&](uint32_t i) { return w_one((double)value(i)); });
+    // Min-p's cut, the first rank below the floor (tested before top-p's at each rank, sample.rs:237-251).
     keep = n;
-    if (tid == 0) {
-      sh.done = 0;
-      sh.sum = 0.0;
-    }
-    __syncthreads();
-    for (uint32_t t0 = 0; t0 < n; t0 += kStage) {
-      const uint32_t c = min((uint32_t)kStage, n - t0);
-      for (uint32_t i = tid; i < c; i += kThreads) {
-        const double v = rv(t0 + i);
-        // -1 marks the first token min-p drops (tested before top-p, sample.rs:237-251).
-        sh.wd[i] = (has_floor && v < floor) ? -1.0 : (p.top_p < 1.0f ? w_one(v) : 0.0);
-      }
-      __syncthreads();
-      if (tid == 0) {
-        double cum = sh.sum;
-        for (uint32_t i = 0; i < c; ++i) {
-          if (sh.wd[i] < 0.0) {
-            sh.keep = t0 + i;
-            sh.done = 1;
-            break;
-          }
-          if (p.top_p < 1.0f) {
-            cum = __dadd_rn(cum, __ddiv_rn(sh.wd[i], total1));
-            if (cum >= top_p) {
-              sh.keep = t0 + i + 1;
-              sh.done = 1;
-              break;
-            }
-          }
+    if (has_floor) {
+      uint32_t first = n;
+      for (uint32_t j = tid; j < n; j += kThreads)
+        if (rv(j) < floor) {
+          first = j;
+          break;
         }
-        sh.sum = cum;
-      }
-      __syncthreads();
-      if (sh.done) break;
+      keep = block_min_u32<kWaves>(first, sh.red_u);
     }
-    if (sh.done) keep = sh.keep;
-    __syncthreads();
+    if (p.top_p < 1.0f) {
+      const double total1 = exact_sum(sh, n, [&](uint32_t i) { return w_one((double)value(i)); });
+      uint32_t first;
+      exact_fold(sh, keep, top_p, true, &first, [&](uint32_t j) { return __ddiv_rn(w_one(rv(j)), total1); });
+      if (first != kNone) keep = first + 1;
+    }
   } else {
     unfiltered = true;
     keep = n;
@@ -298,36 +328,12 @@ __device__ __noinline__ void exact_row(const FinishArgs& a, const RowParams& p, 
   // The draw: u = unit() * total, then the first rank whose cumulative weight exceeds u.
   double total;
   if (unfiltered)
-    total = seq_fold(sh, n, [&](uint32_t i) { return w_temp((double)value(i)); });
+    total = exact_sum(sh, n, [&](uint32_t i) { return w_temp((double)value(i)); });
   else
-    total = seq_fold(sh, keep, [&](uint32_t j) { return w_temp(rv(j)); });
-  const double u = __dmul_rn(sh.u01, total);
-  if (tid == 0) {
-    sh.done = 0;
-    sh.sum = 0.0;
-    sh.pick = keep - 1;  // sample.rs:197, 272, 288: the last kept when u is never passed
-  }
-  __syncthreads();
-  for (uint32_t t0 = 0; t0 < keep; t0 += kStage) {
-    const uint32_t c = min((uint32_t)kStage, keep - t0);
-    for (uint32_t i = tid; i < c; i += kThreads) sh.wd[i] = w_temp(rv(t0 + i));
-    __syncthreads();
-    if (tid == 0) {
-      double cum = sh.sum;
-      for (uint32_t i = 0; i < c; ++i) {
-        cum = __dadd_rn(cum, sh.wd[i]);
-        if (u < cum) {
-          sh.pick = t0 + i;
-          sh.done = 1;
-          break;
-        }
-      }
-      sh.sum = cum;
-    }
-    __syncthreads();
-    if (sh.done) break;
-  }
-  const uint32_t pick = sh.pick;
+    total = exact_sum(sh, keep, [&](uint32_t j) { return w_temp(rv(j)); });
+  uint32_t first;
+  exact_fold(sh, keep, __dmul_rn(sh.u01, total), false, &first, [&](uint32_t j) { return w_temp(rv(j)); });
+  const uint32_t pick = first != kNone ? first : keep - 1;  // sample.rs:197, 272, 288: the last kept when u is never passed
   if (tid == 0) {
     a.tokens[row] = idA[pick];
     a.status[row] = AS_ROW_OK | AS_ROW_EXACT_PATH;
@@ -1340,8 +1346,15 @@ __device__ __forceinline__ void deep_collect(const float* x, const uint32_t* pcn
   });
 }
 
+// What deep_bins came to: the row's bins do not fit its passes (the full deep path may take them), the row is
+// settled, or a decision among the collected values lies inside its bounds: the exact-order path takes it, or
+// (kBinsNeedTotal) the passes run once more with the row's total from exact_total, whose error is most of the
+// bounds of a decision that compares with it (gN: n roundings). An unfiltered 256-row call at 248,320 values
+// had such a row in one call of 140, which the exact-order path took 10 to 20 ms over.
+enum : uint32_t { kBinsNoFit = 0, kBinsDone = 1, kBinsUndecided = 2, kBinsNeedTotal = 3 };
+
 template <bool kDist>
-__device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, uint32_t row, bool pen) {
+__device__ __noinline__ uint32_t deep_bins(const FinishArgs& a, const RowParams& p, uint32_t row, bool pen) {
   constexpr uint32_t kNB = kDist ? as_launch::kDistBins : kDeepBins;
   Shared& sh = shm();
   const uint32_t n = a.n, tid = threadIdx.x;
@@ -1409,7 +1422,7 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
     double* gm = reinterpret_cast<double*>(gc + kNB);
     double* gw = gm + kNB;
     if (!sh.dp_pub) deep_publish_hist(a, row, mk);  // unless the row published it before its candidates
-    if (!deep_run(a, row, 0)) return false;
+    if (!deep_run(a, row, 0)) return kBinsNoFit;
     for (uint32_t b = tid; b < kNB; b += kThreads) {
       hc[b] = ld_agent(gc + b);
       hm[b] = ld_agent(gm + b);
@@ -1438,12 +1451,14 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
   // Inclusive prefixes over the bins, in place: kDPer bins per thread, then the block.
   constexpr int kDPer = kNB / kThreads;
   static_assert(kNB % kThreads == 0, "whole bins per thread");
+  uint32_t c_max = 0;  // the fullest bin's values
   {
     uint32_t c4[kDPer], cs = 0;
     double m4[kDPer], w4[kDPer], ms = 0.0, ws = 0.0;
 #pragma unroll
     for (int q = 0; q < kDPer; ++q) {
       const uint32_t b = tid * kDPer + q;
+      c_max = max(c_max, hc[b]);
       cs += hc[b];
       ms = __dadd_rn(ms, hm[b]);
       ws = __dadd_rn(ws, hw[b]);
@@ -1463,6 +1478,7 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
       hw[b] = __dadd_rn(wb, w4[q]);
     }
   }
+  c_max = block_max_u32<kWaves>(c_max, sh.red_u);
   __syncthreads();
   // Every prefix (and the totals) is within E of the exact sum of the reference's terms: each term is
   // within kPassRel of the reference's and goes through one f64 atomic add and at most
@@ -1473,6 +1489,17 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
   const double g_all = gamma_ub(2.0 * (double)n + 128.0) + kPassRel * (1.0 + 1e-6);
   const double Em = g_all * M_all, Ew = g_all * W_all;
   const double gj = gamma_ub(2.0 * (double)n + 4.0) + 10.0 * kU;
+  // The decisions among the collected values take closer bounds: a prefix of the bins is within eo of the
+  // exact sum of its terms (a bin's terms are added one after another, at most c_max of them and, in a
+  // shared pass, a part's at a time, then through the scans' few adds); the reference's total in index
+  // order is within gN of its terms' exact sum, and its cumulative at rank r folds r + 1 terms, not n.
+  // (At 248,320 values a draw with no filter fell inside the wider bounds in about one call of 40 with 256
+  // rows, and took the full deep path or the exact-order path: 7 to 30 ms.)
+  const double eo = kPassRel * (1.0 + 1e-6) + gamma_ub((double)c_max + (double)as_launch::tail_parts(n) + 128.0);
+  const double gN = gamma_ub((double)n);
+  // The cumulative's bounds at rank r: top-p's quotients and their sum, and the draw's sum.
+  auto rel_p = [](uint32_t r) -> double { return gamma_ub(2.0 * (double)r + 6.0) + 10.0 * kU; };
+  auto rel_d = [](uint32_t r) -> double { return gamma_ub((double)r + 1.0) + 4.0 * kU; };
   auto C = [&](uint32_t b) -> uint32_t { return b == kNone ? 0u : hc[b]; };  // through bin b; kNone: none
   auto Mc = [&](uint32_t b) -> double { return b == kNone ? 0.0 : hm[b]; };
   auto Wc = [&](uint32_t b) -> double { return b == kNone ? 0.0 : hw[b]; };
@@ -1488,7 +1515,7 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
       if (hc[b] >= kk) a0 = min(a0, b);
     }
     bk = block_min_u32<kWaves>(a0, sh.red_u);
-    if (bk == kNone) return false;
+    if (bk == kNone) return kBinsNoFit;
   }
   // top-p's total1: the row's, or the top-k ranks' (those of the bins before bk and some of bk's:
   // bounded here, summed from bk's sorted values below; each bound three times the error of that
@@ -1504,6 +1531,10 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
   // target); at the end of c_hi it has surely been reached (for a top-k row, at bk's end at the
   // latest: past rank k - 1 nothing is kept).
   double tp_lo = top_p * M_lo, tp_hi = top_p * M_hi;
+  // The same among the collected values: the row's total1 closer, or (a top-k row) that of its k ranks once
+  // they are summed, a fold of kk terms within Ek.
+  double tq_lo = top_p * (M_all - (eo + gN) * M_all), tq_hi = top_p * (M_all + (eo + gN) * M_all);
+  const double Ek = (eo + gamma_ub((double)kk) + 2.0 * gamma_n(64.0)) * M_all;
   uint32_t c_lo = kNone, c_hi = kNone;
   if (by_top_p) {
     uint32_t a0 = kNone, a1 = kNone;
@@ -1609,7 +1640,7 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
         ++nr;
       }
     }
-    if (over) return false;
+    if (over) return kBinsNoFit;
   }
   // Per run: the count and weights before it, and where its values start among the collected ones.
   uint32_t cbr[kBinRanges], first[kBinRanges];
@@ -1657,7 +1688,7 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
       }
       __hip_atomic_store(gp(lc), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (!deep_run(a, row, 1)) return false;
+    if (!deep_run(a, row, 1)) return kBinsNoFit;
     if (tid == 0) sh.nsk = ld_agent(lc);
     __syncthreads();
     const uint32_t got = sh.nsk;
@@ -1687,7 +1718,7 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
     for (uint32_t h = tid; h < extra; h += kThreads) hist_two(gload(a.extra_ids + h));
   }
   __syncthreads();
-  if (!fits || sh.pick != collected || collected == 0) return false;
+  if (!fits || sh.pick != collected || collected == 0) return kBinsNoFit;
   // The bucket sort spreads keys below its kmax over its buckets: the collected values' own largest
   // key, since they lie in a few bins far below the row's largest (with that one most would share a
   // few buckets).
@@ -1695,7 +1726,7 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
   for (uint32_t i = tid; i < collected; i += kThreads) ck = max(ck, (uint32_t)(sh.sk[i] >> 32));
   ck = block_max_u32<kWaves>(ck, sh.red_u);
   const uint32_t P = sort_candidates(sh, collected, 0ull, ck, kNone);
-  if (P != collected) return false;
+  if (P != collected) return kBinsNoFit;
   auto val = [&](uint32_t i) -> float { return packed_value(sh.sk[i]); };
   auto run_of = [&](uint32_t i) -> uint32_t { return (i >= first[2]) ? 2u : (i >= first[1] ? 1u : 0u); };
   auto rank_of = [&](uint32_t i, uint32_t k) -> uint32_t { return sel3(k, cbr[0], cbr[1], cbr[2]) + (i - sel3(k, first[0], first[1], first[2])); };
@@ -1720,6 +1751,12 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
   };
   const double g40 = 2.0 * gamma_n(40.0);
 
+  // A row's total in index order (no filter's, or top-p's total1) folded rounding for rounding, once the
+  // caller has it (exact_total): the decisions below then take it in place of the bins' bounds on it.
+  const bool by_total = unfiltered || (need_c && !topk), have_total = sh.ex_have != 0u;
+  const double u_tot = have_total ? __dmul_rn(sh.u01, sh.ex_total) : 0.0;
+  if (have_total) tq_lo = tq_hi = top_p * sh.ex_total;
+  const uint32_t undecided = by_total && !have_total ? kBinsNeedTotal : kBinsUndecided;
   // Up to kWaveMax collected values: wave 0 takes the decisions below from registers (lane l holds
   // collected values kWPer l .. kWPer l + kWPer - 1, their prefixes come from a wave scan) with the
   // same bounds and no block-wide step, and the other waves wait at one barrier. A prefix through
@@ -1783,14 +1820,14 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
       };
       bool ok = true;
       uint32_t keep_w = n, k_floor = kNone;
-      double Wk = W_all, Wk_err = Ew;
+      double Wk = W_all, gk = gN;
       if (need_c || need_f || topk) {
         uint32_t jl = kNone, jh = kNone, jf = kNone;
         if (need_c) {
 #pragma unroll
           for (int q = 0; q < kWPer; ++q) w[q] = i0 + q < P ? w1(v[q]) : 0.0;
           prefixes();
-          double tlo = tp_lo, thi = tp_hi;
+          double tlo = tq_lo, thi = tq_hi;
           if (topk) {
             uint32_t home = kNone;
             const uint32_t j = index_of(kk - 1, &home);
@@ -1798,18 +1835,18 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
               ok = false;
             } else {
               const double Mk = __dadd_rn(sel3(home, mbr[0], mbr[1], mbr[2]), run_part(j, home));
-              tlo = top_p * (Mk - Em2);
-              thi = top_p * (Mk + Em2);
+              tlo = top_p * (Mk - Ek);
+              thi = top_p * (Mk + Ek);
             }
           }
-          const double err = Em + g40 * M_all;
 #pragma unroll
           for (int q = 0; q < kWPer; ++q) {
             if (i0 + q >= P || rk[q] >= kk) continue;
             const uint32_t k = rn[q];
             const double S = __dadd_rn(sel3(k, mbr[0], mbr[1], mbr[2]), __dsub_rn(pre[q], sel3(k, rb[0], rb[1], rb[2])));
-            if ((S + err) * (1.0 + gj) >= tlo) jl = min(jl, rk[q]);
-            if ((S - err) * (1.0 - gj) >= thi) jh = min(jh, rk[q]);
+            const double err = eo * S + g40 * M_all, rel = rel_p(rk[q]);
+            if ((S + err) * (1.0 + rel) >= tlo) jl = min(jl, rk[q]);
+            if ((S - err) * (1.0 - rel) >= thi) jh = min(jh, rk[q]);
           }
         }
 #pragma unroll
@@ -1830,7 +1867,7 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
         }
         if (need_f) k_floor = min(jf, cf_through);
         keep_w = min(min(k_topp, k_floor), kk);
-        Wk_err = Ew + 2.0 * gamma_n(64.0) * W_all;
+        gk = gamma_ub((double)keep_w);
       }
       // The weights at T and their prefixes; the kept weight, a prefix of whole bins when min-p cuts
       // at its bin's ends, else a run's prefix plus its terms through rank keep - 1.
@@ -1850,9 +1887,10 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
         }
       }
       // The draw, as below.
-      const double ulo = sh.u01 * (Wk - Wk_err) * (1.0 - gj) * (1.0 - 4.0 * kU);
-      const double uhi = sh.u01 * (Wk + Wk_err) * (1.0 + gj) * (1.0 + 4.0 * kU);
-      const double err = Ew + g40 * W_all;
+      const double Wk_err = eo * Wk + 2.0 * gamma_n(64.0) * W_all;
+      double ulo = sh.u01 * (Wk - Wk_err) * (1.0 - gk) * (1.0 - 4.0 * kU);
+      double uhi = sh.u01 * (Wk + Wk_err) * (1.0 + gk) * (1.0 + 4.0 * kU);
+      if (have_total && unfiltered) ulo = uhi = u_tot;
       uint32_t jp = kNone, jc = kNone, last = kNone;
 #pragma unroll
       for (int q = 0; q < kWPer; ++q) {
@@ -1860,8 +1898,9 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
         if (rk[q] + 1 == keep_w) last = i0 + q;
         const uint32_t k = rn[q];
         const double S = __dadd_rn(sel3(k, wbr[0], wbr[1], wbr[2]), __dsub_rn(pre[q], sel3(k, rb[0], rb[1], rb[2])));
-        if ((S + err) * (1.0 + gj) > ulo) jp = min(jp, rk[q]);
-        if ((S - err) * (1.0 - gj) > uhi) jc = min(jc, rk[q]);
+        const double err = eo * S + g40 * W_all, rel = rel_d(rk[q]);
+        if ((S + err) * (1.0 + rel) > ulo) jp = min(jp, rk[q]);
+        if ((S - err) * (1.0 - rel) > uhi) jc = min(jc, rk[q]);
       }
       jp = wave_min_u32(jp);
       jc = wave_min_u32(jc);
@@ -1888,7 +1927,7 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
       }
     }
     __syncthreads();
-    return sh.pick != 0;
+    return sh.pick != 0 ? (uint32_t)kBinsDone : undecided;
   }
 
   // The cut (sample.rs:230-252): at the first rank below the floor, or one past the first whose
@@ -1903,26 +1942,26 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
     return block_min_u32<kWaves>(home, sh.red_u);
   };
   uint32_t keep = n;
-  double Wkeep = W_all, Wkeep_err = Ew;
+  double Wkeep = W_all, gk = gN;
   if (need_c || need_f || topk) {
     for (uint32_t i = tid; i < P; i += kThreads) sh.wd[i] = need_c ? w1(val(i)) : 0.0;
     __syncthreads();
+    double tlo = tq_lo, thi = tq_hi;
     if (topk && need_c) {
       // top-p's total1 over the top-k ranks: the prefix before rank k - 1's run plus that run's
       // terms through it, within Em2 of the exact sum; the targets narrow to it.
       const uint32_t home = home_of(kk - 1);
-      if (home == kNone) return false;
+      if (home == kNone) return kBinsUndecided;
       double part = 0.0;
       for (uint32_t i = tid; i < P; i += kThreads)
         if (run_of(i) == home && rank_of(i, home) < kk) part += sh.wd[i];
       part = block_sum_f64<kWaves>(part, sh.red_d);
       const double Mk = __dadd_rn(sel3(home, mbr[0], mbr[1], mbr[2]), part);
-      tp_lo = top_p * (Mk - Em2);
-      tp_hi = top_p * (Mk + Em2);
+      tlo = top_p * (Mk - Ek);
+      thi = top_p * (Mk + Ek);
     }
     scan_runs();
     uint32_t jl = kNone, jh = kNone, jf = kNone;
-    const double err = Em + g40 * M_all;
 #pragma unroll
     for (int q = 0; q < kScanPer; ++q) {
       const uint32_t i = tid * kScanPer + q;
@@ -1932,8 +1971,9 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
       if (need_f && !(val(i) >= floorf)) jf = min(jf, r);
       if (need_c) {
         const double S = __dadd_rn(sel3(k, mbr[0], mbr[1], mbr[2]), __dsub_rn(__dadd_rn(off, loc[q]), run_base[k]));
-        if ((S + err) * (1.0 + gj) >= tp_lo) jl = min(jl, r);
-        if ((S - err) * (1.0 - gj) >= tp_hi) jh = min(jh, r);
+        const double err = eo * S + g40 * M_all, rel = rel_p(r);
+        if ((S + err) * (1.0 + rel) >= tlo) jl = min(jl, r);
+        if ((S - err) * (1.0 - rel) >= thi) jh = min(jh, r);
       }
     }
     jl = block_min_u32<kWaves>(jl, sh.red_u);
@@ -1946,7 +1986,7 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
       if (topk && jl == kNone) {
         k_topp = kNone;
       } else {
-        if (jl != jh || jh == kNone) return false;
+        if (jl != jh || jh == kNone) return undecided;
         k_topp = jh + 1;
       }
     }
@@ -1964,14 +2004,14 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
       Wkeep = wf_before;
     } else {
       const uint32_t home = home_of(keep - 1);
-      if (home == kNone) return false;
+      if (home == kNone) return kBinsUndecided;
       double part = 0.0;
       for (uint32_t i = tid; i < P; i += kThreads)
         if (run_of(i) == home && rank_of(i, home) < keep) part += sh.wd[i];
       part = block_sum_f64<kWaves>(part, sh.red_d);
       Wkeep = __dadd_rn(sel3(home, wbr[0], wbr[1], wbr[2]), part);
     }
-    Wkeep_err = Ew + 2.0 * gamma_n(64.0) * W_all;
+    gk = gamma_ub((double)keep);
   } else {
     for (uint32_t i = tid; i < P; i += kThreads) sh.wd[i] = wt(val(i));
     __syncthreads();
@@ -1980,9 +2020,10 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
   // The draw (sample.rs:260-272, 274-292): u = unit() * (the kept weight), then the first kept rank
   // whose cumulative at T passes u, or the last kept one when none does.
   scan_runs();
-  const double ulo = sh.u01 * (Wkeep - Wkeep_err) * (1.0 - gj) * (1.0 - 4.0 * kU);
-  const double uhi = sh.u01 * (Wkeep + Wkeep_err) * (1.0 + gj) * (1.0 + 4.0 * kU);
-  const double err = Ew + g40 * W_all;
+  const double Wkeep_err = eo * Wkeep + 2.0 * gamma_n(64.0) * W_all;
+  double ulo = sh.u01 * (Wkeep - Wkeep_err) * (1.0 - gk) * (1.0 - 4.0 * kU);
+  double uhi = sh.u01 * (Wkeep + Wkeep_err) * (1.0 + gk) * (1.0 + 4.0 * kU);
+  if (have_total && unfiltered) ulo = uhi = u_tot;
   uint32_t jp = kNone, jc = kNone, last = kNone;
 #pragma unroll
   for (int q = 0; q < kScanPer; ++q) {
@@ -1992,8 +2033,9 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
     if (r >= keep) continue;
     if (r + 1 == keep) last = i;
     const double S = __dadd_rn(sel3(k, wbr[0], wbr[1], wbr[2]), __dsub_rn(__dadd_rn(off, loc[q]), run_base[k]));
-    if ((S + err) * (1.0 + gj) > ulo) jp = min(jp, r);
-    if ((S - err) * (1.0 - gj) > uhi) jc = min(jc, r);
+    const double err = eo * S + g40 * W_all, rel = rel_d(r);
+    if ((S + err) * (1.0 + rel) > ulo) jp = min(jp, r);
+    if ((S - err) * (1.0 - rel) > uhi) jc = min(jc, r);
   }
   jp = block_min_u32<kWaves>(jp, sh.red_u);
   jc = block_min_u32<kWaves>(jc, sh.red_u);
@@ -2003,28 +2045,49 @@ __device__ __noinline__ bool deep_bins(const FinishArgs& a, const RowParams& p, 
   // the first of all.
   uint32_t pick_rank;
   if (jp == kNone) {
-    if (last == kNone) return false;  // the last kept value was not collected
+    if (last == kNone) return kBinsUndecided;  // the last kept value was not collected
     pick_rank = keep - 1;
   } else if (jp == jc) {
     pick_rank = jc;
   } else {
-    return false;
+    return undecided;
   }
   uint32_t pi = kNone;
   for (uint32_t i = tid; i < P; i += kThreads)
     if (rank_of(i, run_of(i)) == pick_rank) pi = i;
   pi = block_min_u32<kWaves>(pi, sh.red_u);
-  if (pi == kNone) return false;
+  if (pi == kNone) return kBinsUndecided;
   if (tid == 0) {
     a.tokens[row] = packed_id(sh.sk[pi]);
     a.status[row] = AS_ROW_OK | AS_ROW_DEEP_PATH;
     if (a.kept_count) a.kept_count[row] = keep;
   }
-  return true;
+  return kBinsDone;
 }
 
 
-// Returns true when it settled the row.
+// sh.ex_total: the reference's total of the row in index order, at T for a row with no filter
+// (sample.rs:274-282), else at T = 1 (total1, sample.rs:218-222), rounding for rounding.
+__device__ __noinline__ void exact_total(const FinishArgs& a, const RowParams& p, uint32_t row, bool pen) {
+  Shared& sh = shm();
+  const uint32_t* cnt = a.scratch + (uint64_t)row * a.scratch_stride;
+  const float* x = a.logits + (uint64_t)row * a.row_stride;
+  const double top = (double)key_value(sh.mk), temp = (double)p.temp;
+  const bool at_t = !(p.top_p < 1.0f);
+  const double s = exact_sum(sh, a.n, [&](uint32_t i) -> double {
+    float v = gload(x + i);
+    const uint32_t c = pen ? gload(cnt + i) : 0u;
+    if (c) v = penalize_out(v, c, p);
+    const double d = __dsub_rn((double)v, top);
+    return as_exp::exp_with(sh.tab, at_t ? __ddiv_rn(d, temp) : d);
+  });
+  if (threadIdx.x == 0) {
+    sh.ex_total = s;
+    sh.ex_have = 1;
+  }
+  __syncthreads();
+}
+
 // The row's history counts in its scratch (u32 per id), for the passes over the whole row: whether
 // penalties act (false: no counts).
 __device__ __noinline__ bool deep_prep(const FinishArgs& a, const RowParams& p, uint32_t row) {
@@ -3132,6 +3195,7 @@ __device__ __forceinline__ void finish_row(const FinishArgs& a, uint32_t row) {
     sh.tail_listed = 0;
     sh.tail_parts = 0;
     sh.dp_pub = 0;
+    sh.ex_have = 0;
   }
   const bool draws = p.mode != kModeGreedy;
   uint64_t s4[4] = {0ull, 0ull, 0ull, 0ull};
@@ -3645,12 +3709,17 @@ __device__ __forceinline__ void finish_row(const FinishArgs& a, uint32_t row) {
     if (sh.tail_slot != kNone && !sh.tail_waited) tail_wait(a, row);
     const RowParams& pr = a.params[row];
     const bool pen = deep_prep(a, pr, row);
-    bool done = false;
+    uint32_t bins = kBinsNoFit;
     if (!sh.stats_bad && !a.kept_ids) {
-      done = a.deep_help ? deep_bins<true>(a, pr, row, pen) : deep_bins<false>(a, pr, row, pen);
+      bins = a.deep_help ? deep_bins<true>(a, pr, row, pen) : deep_bins<false>(a, pr, row, pen);
       __syncthreads();
+      if (bins == kBinsNeedTotal) {
+        exact_total(a, pr, row, pen);
+        bins = deep_bins<false>(a, pr, row, pen);
+        __syncthreads();
+      }
     }
-    if (!done && !deep_row(a, pr, row, pen)) {
+    if (bins == kBinsUndecided || (bins == kBinsNoFit && !deep_row(a, pr, row, pen))) {
       __syncthreads();
       exact_row(a, pr, row);
     }
