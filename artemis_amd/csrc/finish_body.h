@@ -610,7 +610,8 @@ __device__ __forceinline__ uint32_t decide_draw(Shared& sh, uint32_t m, const do
 // On success the row's kept count (or P, a lower bound, with AS_ROW_KEPT_PARTIAL) and status are
 // returned and sh.pick / sh.sum hold the rank drawn and the total.
 __device__ __forceinline__ bool fast_partial(const FinishArgs& a, Shared& sh, const RowParams& p, uint32_t P,
-                                             bool floor_cut, uint32_t* keep_out, uint32_t* status_out) {
+                                             bool floor_cut, uint32_t* keep_out, uint32_t* status_out,
+                                             bool* past_out) {
   const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave, n = a.n;
   const double top = (double)key_value(sh.mk), temp = (double)p.temp, top_p = (double)p.top_p;
   const bool has_floor = p.min_p > 0.0f, topp = p.top_p < 1.0f;
@@ -755,6 +756,9 @@ __device__ __forceinline__ bool fast_partial(const FinishArgs& a, Shared& sh, co
       const bool more = pick == kNone && past_mw && ((kk != kNone && kk == m) || past) && m > kWaveMax;
       sh.fp_m = more ? m : 0u;
       sh.fp_past = past ? 1u : 0u;
+      sh.x1 = X;
+      sh.eps1 = eps;
+      sh.r_prefix = S1;
       sh.fp_lo = ulo;
       sh.fp_hi = uhi;
     }
@@ -775,7 +779,10 @@ __device__ __forceinline__ bool fast_partial(const FinishArgs& a, Shared& sh, co
     __syncthreads();
     keep = sh.keep;
   }
-  if (keep == kNone) return false;
+  if (keep == kNone) {
+    *past_out = sh.fp_past != 0u;
+    return false;
+  }
   *keep_out = keep;
   *status_out = keep == P && !(im_exact || P == n) ? (uint32_t)AS_ROW_KEPT_PARTIAL : (uint32_t)AS_ROW_OK;
   return true;
@@ -3388,13 +3395,13 @@ __device__ __forceinline__ void finish_row(const FinishArgs& a, uint32_t row) {
     if (tid == 0) sh.prefix = P;
     uint32_t keep = kNone;
     uint32_t status = AS_ROW_OK;
-    bool drawn = false;
+    bool drawn = false, past = false;
     // A row without a top-k and without kept lists first takes the fast decision, and a flagged row
     // waits for S's sums only when that does not settle it. A flagged row whose floor set is not vast
     // skips it: min-p cuts first within S, and the draw needs S's values.
     if (p.mode == kModePartial && (p.top_p < 1.0f || has_floor) && !a.kept_ids && !too_many && P > 0 &&
         P + kWaveMax <= (uint32_t)kCap && (sh.tail_slot == kNone || sh.vast))
-      drawn = fast_partial(a, sh, p, P, floor_cut, &keep, &status);
+      drawn = fast_partial(a, sh, p, P, floor_cut, &keep, &status, &past);
     // S's listed values past the sorted candidates, not yet sorted (sorted only when the draw lands
     // past the candidates, or kept lists need them): how many, and where they start.
     uint32_t tail_unsorted = 0, sorted_p = 0;
@@ -3439,6 +3446,26 @@ __device__ __forceinline__ void finish_row(const FinishArgs& a, uint32_t row) {
       // A top-k row's k best are among the sorted values only when at least k rank at or above R.
       const bool short_topk = p.mode == kModeTopK && P < p.top_k;
 
+      // The draw past the sorted values, whose own bounds gave j: undecided, one pass over the row for S's
+      // sums, unless the row has them. With the deep passes shared (a small batch), a row they would settle
+      // takes them at once rather than one workgroup's pass over the row first.
+      auto past_sorted = [&](uint32_t j) {
+        if (j == kNone && !sh.have_tail && !a.deep_help &&
+            tail_sums(a, a.params[row], row, R, has_floor ? floor_f32(floor) : -__builtin_inff(), key_value(sh.mk))) {
+          status |= AS_ROW_TAIL_PASS;
+          j = draw_past(a, a.params[row], row, P, true, false);
+        }
+        if (j != kNone && j < P) {
+          if (tid == 0) sh.pick = j;  // sh.sum holds the sorted weight
+          drawn = true;
+          keep = P;  // a lower bound: the kept set's full size is not known
+          status |= AS_ROW_KEPT_PARTIAL;
+        } else {
+          keep = kNone;
+        }
+        __syncthreads();
+      };
+
       double r_prefix = 0.0;  // the top-p scan's sum of exp(l - top) over the P sorted values
       double x1 = 0.0, eps1 = 0.0;  // total1 and its bound
       if (floor_set) {
@@ -3446,6 +3473,12 @@ __device__ __forceinline__ void finish_row(const FinishArgs& a, uint32_t row) {
         status |= AS_ROW_TAIL_PASS;
       } else if (short_topk || too_many) {
         keep = kNone;
+      } else if (past && sh.tail_slot == kNone) {
+        // fast_partial has tried draw_past's bounds on the sorted values: finding the cut and the draw
+        // from them once more would settle nothing. (248,320 values, top-p 0.95: six rows of a verify call 109.4 us
+        // with the second try, 98.8 without; 256 rows
+        // 365.6 and 353.2.)
+        past_sorted(kNone);
       } else if (p.mode == kModeTopK) {
         // draw_full_sort over the k best (sample.rs:157-197), on wave 0 from registers: top-p's cut,
         // min-p's floor (the ranks are sorted, so it keeps a prefix) and the draw, each decided by
@@ -3548,32 +3581,9 @@ __device__ __forceinline__ void finish_row(const FinishArgs& a, uint32_t row) {
             sh.r_prefix = r_prefix;
           }
           __syncthreads();
-          // S's sums when the row was flagged; else the sorted values alone first, and one
-          // pass over the row when they cannot settle the draw.
-          uint32_t j;
-          if (sh.have_tail) {
-            status |= AS_ROW_TAIL_PASS;
-            j = draw_past(a, a.params[row], row, P, true, true);
-          } else {
-            j = draw_past(a, a.params[row], row, P, false, false);
-            // With the deep passes shared (a small batch), a row they would settle takes them at once
-            // rather than one workgroup's pass over the row first.
-            if (j == kNone && !a.deep_help &&
-                tail_sums(a, a.params[row], row, R, has_floor ? floor_f32(floor) : -__builtin_inff(),
-                          key_value(sh.mk))) {
-              status |= AS_ROW_TAIL_PASS;
-              j = draw_past(a, a.params[row], row, P, true, false);
-            }
-          }
-          if (j != kNone && j < P) {
-            if (tid == 0) sh.pick = j;  // sh.sum holds the sorted weight
-            drawn = true;
-            keep = P;  // a lower bound: the kept set's full size is not known
-            status |= AS_ROW_KEPT_PARTIAL;
-          } else {
-            keep = kNone;
-          }
-          __syncthreads();
+          // S's sums when the row was flagged; else the sorted values alone first.
+          if (sh.have_tail) status |= AS_ROW_TAIL_PASS;
+          past_sorted(draw_past(a, a.params[row], row, P, sh.have_tail != 0u, sh.have_tail != 0u));
         } else {
           keep = kNone;
         }
