@@ -3476,8 +3476,7 @@ __device__ __forceinline__ void finish_row(const FinishArgs& a, uint32_t row) {
       } else if (past && sh.tail_slot == kNone) {
         // fast_partial has tried draw_past's bounds on the sorted values: finding the cut and the draw
         // from them once more would settle nothing. (248,320 values, top-p 0.95: six rows of a verify call 109.4 us
-        // with the second try, 98.8 without; 256 rows
-        // 365.6 and 353.2.)
+        // with the second try, 98.8 without; 256 rows 365.6 and 353.2.)
         past_sorted(kNone);
       } else if (p.mode == kModeTopK) {
         // draw_full_sort over the k best (sample.rs:157-197), on wave 0 from registers: top-p's cut,
