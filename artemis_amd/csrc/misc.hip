@@ -100,17 +100,18 @@ __global__ __launch_bounds__(kArgThreads) void argmax_kernel(const float* __rest
     }
     tail = b0 + 4 * groups;
   }
-  for (uint32_t i0 = tail + tid; i0 < b1; i0 += kArgLoads * kArgThreads) {
+  // (In 64 bits: a slice may end within one step of 2^32.)
+  for (uint64_t i0 = (uint64_t)tail + tid; i0 < b1; i0 += kArgLoads * kArgThreads) {
     float q[kArgLoads];
 #pragma unroll
     for (uint32_t u = 0; u < kArgLoads; ++u) {
-      const uint32_t i = i0 + u * kArgThreads;
+      const uint64_t i = i0 + u * kArgThreads;
       if (i < b1) q[u] = src[i];
     }
 #pragma unroll
     for (uint32_t u = 0; u < kArgLoads; ++u) {
-      const uint32_t i = i0 + u * kArgThreads;
-      if (i < b1) see(q[u], i);
+      const uint64_t i = i0 + u * kArgThreads;
+      if (i < b1) see(q[u], (uint32_t)i);
     }
   }
   uint64_t key = wave_max_u64(bi == kNone ? 0ull : pack(total_key(bv == 0.0f ? 0.0f : bv), bi));

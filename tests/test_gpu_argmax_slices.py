@@ -46,3 +46,25 @@ def test_slices_give_the_twins_pick(n, rows, pad):
         assert got.tolist() == [0xFFFFFFFF if w is None else w for w in want]
         assert addr.tolist() == [(1 << 33) + (0 if w is None else w) * 210 for w in want]
     ctx.close()
+
+
+@pytest.mark.parametrize("skew", [0, 1])
+def test_a_row_that_ends_within_a_step_of_2_to_the_32(skew):
+    # 1,500 short of 2^32: a thread's next index past the row's end does not fit 32 bits. skew 1: the row is
+    # not 16-byte aligned and takes the scalar loads.
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from artemis_amd import Context
+    n = (1 << 32) - 1500
+    if torch.cuda.mem_get_info()[0] < 6 * n:
+        pytest.skip("less than 24 GiB of memory free")
+    dev = torch.device("cuda")
+    x = torch.full((n + 4,), -1.0, dtype=torch.float32, device=dev)[skew:skew + n]
+    ids = torch.empty(1, dtype=torch.int32, device=dev)
+    out = torch.empty(1, dtype=torch.int64, device=dev)
+    ctx = Context(max_rows=1, max_vocab=16)
+    for at, v in ((0, 0.0), (n - 1, 2.0), (n // 2, 2.0)):  # each the row's largest, the last one by a tie
+        x[at] = v
+        ctx.argmax_rows(x, ids, out, 0, 4)
+        assert (int(ids.item()) & 0xFFFFFFFF, int(out.item())) == (at, 4 * at)
+    ctx.close()
