@@ -577,9 +577,16 @@ int as_argmax_rows(as_ctx* c, const float* logits, uint64_t row_stride, uint32_t
     return fail(c, AS_ERR_INVALID, "as_argmax_rows: bad pointers or row_stride < n");
   AS_HIP(c, hipSetDevice(c->device));
   const bool vec = aligned16(logits) && (row_stride % 4 == 0);
+  // Rows in slices meet in the context's scratch, which one call at a time may use: the stream orders them.
+  // A captured call may be replayed on any stream, beside other calls and after as_destroy, and a per-thread
+  // stream orders one thread's calls only: those take no scratch.
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  const hipError_t ce = hipStreamIsCapturing(c->stream, &capture);
+  if (ce != hipSuccess) (void)hipGetLastError();  // the legacy stream beside a capture: the launch below tells
+  const bool ordered = ce == hipSuccess && capture == hipStreamCaptureStatusNone && c->stream != hipStreamPerThread;
   uint32_t* arrived = reinterpret_cast<uint32_t*>(c->d_arg + 2 * as_launch::kArgGroups);
-  AS_HIP(c, as_launch::argmax_rows(c->stream, vec, logits, row_stride, n, n_rows, c->d_arg, arrived, ids,
-                                   rows_out, embd, row_bytes, slot));
+  AS_HIP(c, as_launch::argmax_rows(c->stream, vec, logits, row_stride, n, n_rows, ordered ? c->d_arg : nullptr,
+                                   arrived, ids, rows_out, embd, row_bytes, slot));
   return AS_OK;
 }
 

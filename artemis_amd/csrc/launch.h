@@ -203,8 +203,9 @@ hipError_t head_argmax(hipStream_t stream, const void* w, uint32_t wtype, uint64
 hipError_t embed_rows(hipStream_t stream, const uint64_t* rows, uint32_t wtype, uint32_t n, float* y,
                       uint32_t n_tokens);
 
-// best: 2 * kArgGroups u64 of scratch; arrived: kArgGroups u32, zero before the call and after it (rows
-// in slices count their slices there).
+// best: 2 * kArgGroups u64 of scratch, which no other call may use meanwhile, or null: each row is one
+// workgroup's then, and nothing outlives the launch. arrived: kArgGroups u32, zero before the call and
+// after it (rows in slices count their slices there).
 constexpr uint32_t kArgGroups = 768;
 hipError_t argmax_rows(hipStream_t stream, bool vec, const float* logits, uint64_t row_stride,
                        uint32_t n, uint32_t n_rows, uint64_t* best, uint32_t* arrived, uint32_t* ids,

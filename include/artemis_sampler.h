@@ -136,8 +136,9 @@ int as_verify(as_ctx* ctx, const float* rows, uint64_t row_stride, uint32_t n_vo
 
 /* argmax_rows (crates/kernels/src/dispatch.rs:121-153, shaders/argmax_rows.comp): for each of
  * n_rows rows, ids[slot + r] = the largest finite value's index (ties to the lower index) or
- * AS_NO_DRAFT, rows_out[slot + r] = embd + id * row_bytes (id 0 for AS_NO_DRAFT). Stream-ordered;
- * calls on one context must not overlap (they share its scratch). */
+ * AS_NO_DRAFT, rows_out[slot + r] = embd + id * row_bytes (id 0 for AS_NO_DRAFT). Stream-ordered. A
+ * captured call uses none of the context's memory: its graph may be replayed on any stream, beside other
+ * calls and after as_destroy. */
 int as_argmax_rows(as_ctx* ctx, const float* logits, uint64_t row_stride, uint32_t n,
                    uint32_t n_rows, uint32_t* ids, uint64_t* rows_out, uint64_t embd,
                    uint32_t row_bytes, uint32_t slot);
