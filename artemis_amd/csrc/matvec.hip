@@ -8,13 +8,14 @@
 // (tree32.glsl; twin/mod.rs:15-25). The library is built without contraction, so every product is
 // rounded before its add, as the reference's `precise` arithmetic is.
 //
-// F32, BF16 and Q8_0 (matvec_kernel): on CDNA4 a wave of 64 lanes holds two 32-lane row groups (a 32-lane
-// xor shuffle stays inside its half); each group computes two rows per step, so that two units' loads are
-// in flight per lane, and a 256-thread workgroup walks 16-row steps grid-stride, with a grid that fits the
+// F32, BF16, Q8_0 and some Q6_K tables (matvec_kernel): on CDNA4 a wave of 64 lanes holds two 32-lane row
+// groups (a 32-lane xor shuffle stays inside its half); each group computes two rows per step, so that two
+// units' loads are in flight per lane, and a 256-thread workgroup walks 16-row steps grid-stride, with a grid that fits the
 // chip in one round. x is staged once per workgroup in LDS, unit u at xs[33 u ..] (the pad of one float
 // puts the 32 lanes' reads of 32 different units in 32 different banks). Weights are read once, straight
 // from HBM; the compiler merges a unit's 2-byte reads into 16-byte loads (the target allows unaligned
-// global access, and Q8_0's 34-byte blocks are only 2-byte aligned). The K-quants take quad_kernel, below.
+// global access, and Q8_0's 34-byte and Q6_K's 210-byte blocks are only 2-byte aligned). The K-quants take
+// quad_kernel, below, but for the Q6_K tables that row_threads names.
 //
 // head_argmax: the same rows with argmax_rows' epilogue (crates/kernels/shaders/argmax_rows.comp):
 // the largest finite output, ties to the lower index (-0 and +0 tie), computed as the outputs are
@@ -47,6 +48,14 @@ __device__ __forceinline__ uint32_t byte_of(const uint32_t (&q)[8], uint32_t l) 
   return (q[l >> 2] >> (8 * (l & 3))) & 0xFFu;
 }
 
+// Four 6-bit quants q = lo + 16 hi at once, one a byte (lo: the low nibbles of l's bytes, hi: the low pairs of
+// h's), each byte holding q - 32 as a signed byte: lo in its low nibble and hi - 2 (mod 16) in its high one,
+// which v_perm_b32 looks up per byte (byte hi of 0x1000F0E0: 0xE0, 0xF0, 0x00, 0x10). Each value is then one
+// sign-extending byte-to-float conversion; float(q - 32) is exactly the reference's float(q) - 32.
+__device__ __forceinline__ uint32_t q6_bytes(uint32_t l, uint32_t h) {
+  return (l & 0x0F0F0F0Fu) | __builtin_amdgcn_perm(0u, 0x1000F0E0u, h & 0x03030303u);
+}
+
 // quant.glsl unit_dot (twin/matvec.rs:21-84) for unit u of the row; x: the unit's 32 inputs in LDS.
 template <uint32_t kType>
 __device__ __forceinline__ float unit_dot(const uint8_t* __restrict__ row, uint32_t u, const float* x) {
@@ -71,8 +80,7 @@ __device__ __forceinline__ float unit_dot(const uint8_t* __restrict__ row, uint3
       s = s + __uint_as_float(wv[i] & 0xFFFF0000u) * x[2 * i + 1];
     }
     return s;
-  } else {
-    static_assert(kType == AS_WTYPE_Q8_0, "the K-quants take quad_kernel");
+  } else if constexpr (kType == AS_WTYPE_Q8_0) {
     const uint16_t* b = reinterpret_cast<const uint16_t*>(row + 34u * u);
     uint32_t q[8];
     load32(b + 1, q);
@@ -81,6 +89,28 @@ __device__ __forceinline__ float unit_dot(const uint8_t* __restrict__ row, uint3
 #pragma unroll
     for (int i = 0; i < 32; ++i) s = s + (float)(int8_t)byte_of(q, i) * x[i];
     return d * s;
+  } else {
+    // Q6_K: unit j of a block is half n = j / 4, quarter m = j % 4.
+    static_assert(kType == AS_WTYPE_Q6_K, "Q4_K and Q5_K take quad_kernel");
+    const uint16_t* b = reinterpret_cast<const uint16_t*>(row + 210u * (u / 8));
+    const uint32_t j = u % 8, n = j / 4, m = j % 4;
+    uint32_t ql[8], qh[8];
+    load32(b + 32 * n + 16 * (m & 1), ql);
+    load32(b + 64 + 16 * n, qh);
+    const uint32_t scs = b[96 + 4 * n + m], dh = b[104];
+    float sa = 0.0f, sb = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t s4 = q6_bytes(ql[i] >> (4 * (m >> 1)), qh[i] >> (2 * m));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float prod = (float)(int8_t)(uint8_t)(s4 >> (8 * e)) * x[4 * i + e];
+        if (i < 4) sa = sa + prod;
+        else sb = sb + prod;
+      }
+    }
+    const float pa = (float)(int8_t)(scs & 0xFFu) * sa, pb = (float)(int8_t)(scs >> 8) * sb;
+    return half_u16(dh) * (pa + pb);
   }
 }
 
@@ -246,16 +276,12 @@ struct Quad<AS_WTYPE_Q6_K, kWords> {
 #pragma unroll
     for (int m = 0; m < 4; ++m) sa[m] = sb[m] = 0.0f;
   }
-  // Values 4i .. 4i + 3 of the four units. Four 6-bit quants q = lo + 16 hi at once, one a byte, each byte
-  // holding q - 32 as a signed byte: lo in its low nibble and hi - 2 (mod 16) in its high one, which
-  // v_perm_b32 looks up per byte (byte hi of 0x1000F0E0: 0xE0, 0xF0, 0x00, 0x10). Each value is then one
-  // sign-extending byte-to-float conversion; float(q - 32) is exactly the reference's float(q) - 32.
+  // Values 4i .. 4i + 3 of the four units.
   __device__ __forceinline__ void step(int i, const f32x4 (&x)[4]) {
     const uint32_t h = high(i), l0 = low(i), l1 = low(8 + i);
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-      const uint32_t hi = __builtin_amdgcn_perm(0u, 0x1000F0E0u, (h >> (2 * m)) & 0x03030303u);
-      const uint32_t s4 = (((m & 1 ? l1 : l0) >> (4 * (m >> 1))) & 0x0F0F0F0Fu) | hi;
+      const uint32_t s4 = q6_bytes((m & 1 ? l1 : l0) >> (4 * (m >> 1)), h >> (2 * m));
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float prod = (float)(int8_t)(uint8_t)(s4 >> (8 * e)) * x[m][e];
@@ -454,6 +480,28 @@ uint32_t grid_for(K kernel, size_t lds, uint32_t rows, uint32_t step) {
   return (uint32_t)(g < n_steps ? g : n_steps);
 }
 
+// A K-quant row's threads: 4, 8 or 16 of quad_kernel's, or 32, a unit per lane (matvec_kernel; Q6_K only).
+//  - Up to 4 quads, 4 threads hold the row whole (its first 16 partials, the others +0.0): 16 would leave 12
+//    idle (Q4_K, 120,000 x 512: 9.7 us against 30.9, and 26.9 for a unit per lane). Up to 8, 8 threads do, in
+//    one step (248,320 x 1,024: Q5_K 32.0 us against 57.1 with 16, Q6_K 37.0 against 67.4 and 49.3 for a unit
+//    per lane).
+//  - Longer rows take the quads in steps of 8 or 16 threads. 16 leave half a step or more idle when the last
+//    step holds 8 quads or fewer; 8 do not, but need 16,384 rows for two waves per SIMD, without which each
+//    step's loads are waited for (2,560 values, 65,536 and 8,192 rows, 8 against 16 threads: Q5_K 26.6 and
+//    31.4 us, 8.3 and 7.6). Elsewhere 16 measured best for Q5_K and Q6_K (238,095 x 2,048: Q6_K 82.7 against
+//    93.0), and 8 for Q4_K, whose weights cost the fewest instructions beside the tree that half as many
+//    threads share (248,320 x 2,048: 52.8 against 57.8).
+//  - Q6_K between the two, where 16 threads idle and rows are few: a unit per lane, which fills its 32 lanes
+//    (2,560 values: 6,144 rows 7.6 us, against 7.9 with 8 threads and 8.0 with 16; 20,480 rows 14.4 against 15.5 and
+//    15.5; 32,768 rows 20.9 against 20.1 with 8).
+uint32_t row_threads(uint32_t wtype, uint32_t quads, uint32_t rows) {
+  if (quads <= 4) return 4;
+  if (quads <= 8) return 8;
+  const bool half_idle = quads % 16 != 0 && quads % 16 <= 8;
+  if (wtype == AS_WTYPE_Q6_K) return !half_idle ? 16 : (rows < 32768 ? 32 : 8);
+  return rows >= 16384 && (half_idle || wtype == AS_WTYPE_Q4_K) ? 8 : 16;
+}
+
 template <bool kArgmax>
 hipError_t launch(hipStream_t stream, const void* w, uint32_t wtype, uint64_t row_bytes, uint32_t rows, uint32_t k,
                   const float* x, float* y, uint64_t* partials, uint32_t* groups) {
@@ -461,42 +509,42 @@ hipError_t launch(hipStream_t stream, const void* w, uint32_t wtype, uint64_t ro
   const size_t qlds = (size_t)(k / 128) * (kQuadStride + 4) * sizeof(float);
   const uint8_t* wb = static_cast<const uint8_t*>(w);
   const dim3 block(kThreads);
+  const uint32_t threads = row_threads(wtype, k / 128, rows);
   switch (wtype) {
-#define AS_MV(T)                                                                                                     \
-  case T: {                                                                                                          \
+#define AS_MV_RUN(T)                                                                                                 \
+  {                                                                                                                  \
     *groups = grid_for(matvec_kernel<T, kArgmax>, lds, rows, kRowsPerStep);                                          \
     hipLaunchKernelGGL((matvec_kernel<T, kArgmax>), dim3(*groups), block, lds, stream, wb, row_bytes, rows, k, x, y, \
                        partials);                                                                                    \
     break;                                                                                                           \
   }
+#define AS_MV(T) case T: AS_MV_RUN(T)
     AS_MV(AS_WTYPE_F32)
     AS_MV(AS_WTYPE_BF16)
     AS_MV(AS_WTYPE_Q8_0)
-#undef AS_MV
 #define AS_QUAD_T(T, W, N)                                                                                           \
   {                                                                                                                  \
     *groups = grid_for(quad_kernel<T, W, N, kArgmax>, qlds, rows, kThreads / N);                                     \
     hipLaunchKernelGGL((quad_kernel<T, W, N, kArgmax>), dim3(*groups), block, qlds, stream, wb, row_bytes, rows, k,  \
                        x, y, partials);                                                                              \
-  }
-// A row's threads: 4 hold a row of up to four quads (its first 16 partials, the others +0.0) whole, where 16
-// would leave 12 idle (Q4_K, 120,000 x 512: 9.7 us against 30.9, and 26.9 for a unit per lane). Longer rows
-// take the 16 threads that measured best at 248,320 x 2,048 for Q5_K and Q6_K (71.5 against 72.5 us with 8,
-// 89.8 against 97.2), and 8 for Q4_K (61.7 against 66.0), whose weights cost the fewest instructions beside
-// the tree that half as many threads share.
-#define AS_QUAD(T, W, N)                                                                                             \
-  {                                                                                                                  \
-    if (k <= 512) AS_QUAD_T(T, W, 4)                                                                                 \
-    else AS_QUAD_T(T, W, N)                                                                                          \
     break;                                                                                                           \
   }
-    case AS_WTYPE_Q4_K: AS_QUAD(AS_WTYPE_Q4_K, false, 8)
-    case AS_WTYPE_Q5_K: AS_QUAD(AS_WTYPE_Q5_K, false, 16)
+#define AS_QUAD(T, W)                                                                                                \
+  {                                                                                                                  \
+    if (threads == 4) AS_QUAD_T(T, W, 4)                                                                             \
+    if (threads == 8) AS_QUAD_T(T, W, 8)                                                                             \
+    AS_QUAD_T(T, W, 16)                                                                                              \
+  }
+    case AS_WTYPE_Q4_K: AS_QUAD(AS_WTYPE_Q4_K, false)
+    case AS_WTYPE_Q5_K: AS_QUAD(AS_WTYPE_Q5_K, false)
     case AS_WTYPE_Q6_K:
-      if ((uintptr_t)w % 4 == 0) AS_QUAD(AS_WTYPE_Q6_K, true, 16)
-      else AS_QUAD(AS_WTYPE_Q6_K, false, 16)
+      if (threads == 32) AS_MV_RUN(AS_WTYPE_Q6_K)
+      if ((uintptr_t)w % 4 == 0) AS_QUAD(AS_WTYPE_Q6_K, true)
+      AS_QUAD(AS_WTYPE_Q6_K, false)
 #undef AS_QUAD
 #undef AS_QUAD_T
+#undef AS_MV
+#undef AS_MV_RUN
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
