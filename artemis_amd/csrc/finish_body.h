@@ -1354,10 +1354,10 @@ __device__ __forceinline__ void deep_collect(const float* x, const uint32_t* pcn
 }
 
 // What deep_bins came to: the row's bins do not fit its passes (the full deep path may take them), the row is
-// settled, or a decision among the collected values lies inside its bounds: the exact-order path takes it, or
-// (kBinsNeedTotal) the passes run once more with the row's total from exact_total, whose error is most of the
-// bounds of a decision that compares with it (gN: n roundings). An unfiltered 256-row call at 248,320 values
-// had such a row in one call of 140, which the exact-order path took 10 to 20 ms over.
+// settled, or a decision among the collected values lies inside its bounds: the exact-order path takes it, or,
+// when the decision compares with the row's total (an unfiltered row's draw, the cut of a top-p row without a
+// top-k), the passes run once more with the total from exact_total, whose error is most of that decision's
+// bounds (gN: n roundings).
 enum : uint32_t { kBinsNoFit = 0, kBinsDone = 1, kBinsUndecided = 2, kBinsNeedTotal = 3 };
 
 template <bool kDist>
@@ -1760,10 +1760,12 @@ __device__ __noinline__ uint32_t deep_bins(const FinishArgs& a, const RowParams&
 
   // A row's total in index order (no filter's, or top-p's total1) folded rounding for rounding, once the
   // caller has it (exact_total): the decisions below then take it in place of the bins' bounds on it.
-  const bool by_total = unfiltered || (need_c && !topk), have_total = sh.ex_have != 0u;
+  const bool have_total = sh.ex_have != 0u;
   const double u_tot = have_total ? __dmul_rn(sh.u01, sh.ex_total) : 0.0;
   if (have_total) tq_lo = tq_hi = top_p * sh.ex_total;
-  const uint32_t undecided = by_total && !have_total ? kBinsNeedTotal : kBinsUndecided;
+  // What an open cut or an open draw comes to: the total settles only what is compared with it.
+  const uint32_t cut_open = need_c && !topk && !have_total ? kBinsNeedTotal : kBinsUndecided;
+  const uint32_t draw_open = unfiltered && !have_total ? kBinsNeedTotal : kBinsUndecided;
   // Up to kWaveMax collected values: wave 0 takes the decisions below from registers (lane l holds
   // collected values kWPer l .. kWPer l + kWPer - 1, their prefixes come from a wave scan) with the
   // same bounds and no block-wide step, and the other waves wait at one barrier. A prefix through
@@ -1825,7 +1827,8 @@ __device__ __noinline__ uint32_t deep_bins(const FinishArgs& a, const RowParams&
           if ((uint32_t)q == qj) y = pre[q];
         return __dsub_rn(wave_lane_f64(y, j / kWPer), sel3(k, rb[0], rb[1], rb[2]));
       };
-      bool ok = true;
+      uint32_t res = kBinsDone;
+      auto open = [&](uint32_t r) { res = res == kBinsDone ? r : res; };  // the first open decision counts
       uint32_t keep_w = n, k_floor = kNone;
       double Wk = W_all, gk = gN;
       if (need_c || need_f || topk) {
@@ -1839,7 +1842,7 @@ __device__ __noinline__ uint32_t deep_bins(const FinishArgs& a, const RowParams&
             uint32_t home = kNone;
             const uint32_t j = index_of(kk - 1, &home);
             if (j == kNone) {
-              ok = false;
+              open(kBinsUndecided);
             } else {
               const double Mk = __dadd_rn(sel3(home, mbr[0], mbr[1], mbr[2]), run_part(j, home));
               tlo = top_p * (Mk - Ek);
@@ -1867,7 +1870,7 @@ __device__ __noinline__ uint32_t deep_bins(const FinishArgs& a, const RowParams&
           if (topk && jl == kNone) {
             k_topp = kNone;
           } else if (jl != jh || jh == kNone) {
-            ok = false;
+            open(cut_open);
           } else {
             k_topp = jh + 1;
           }
@@ -1889,7 +1892,7 @@ __device__ __noinline__ uint32_t deep_bins(const FinishArgs& a, const RowParams&
         } else {
           uint32_t home = kNone;
           const uint32_t j = keep_w > 0 ? index_of(keep_w - 1, &home) : kNone;
-          if (j == kNone) ok = false;
+          if (j == kNone) open(kBinsUndecided);
           else Wk = __dadd_rn(sel3(home, wbr[0], wbr[1], wbr[2]), run_part(j, home));
         }
       }
@@ -1914,27 +1917,27 @@ __device__ __noinline__ uint32_t deep_bins(const FinishArgs& a, const RowParams&
       last = wave_min_u32(last);
       uint32_t pick_rank = kNone;
       if (jp == kNone) {
-        if (last == kNone) ok = false;
+        if (last == kNone) open(kBinsUndecided);
         else pick_rank = keep_w - 1;
       } else if (jp == jc) {
         pick_rank = jc;
       } else {
-        ok = false;
+        open(draw_open);
       }
       uint32_t home = kNone;
-      const uint32_t pi = ok ? index_of(pick_rank, &home) : kNone;
-      if (pi == kNone) ok = false;
+      const uint32_t pi = res == kBinsDone ? index_of(pick_rank, &home) : kNone;
+      if (pi == kNone) open(kBinsUndecided);
       if (tid == 0) {
-        if (ok) {
+        if (res == kBinsDone) {
           a.tokens[row] = packed_id(sh.sk[pi]);
           a.status[row] = AS_ROW_OK | AS_ROW_DEEP_PATH;
           if (a.kept_count) a.kept_count[row] = keep_w;
         }
-        sh.pick = ok ? 1u : 0u;
+        sh.pick = res;
       }
     }
     __syncthreads();
-    return sh.pick != 0 ? (uint32_t)kBinsDone : undecided;
+    return sh.pick;
   }
 
   // The cut (sample.rs:230-252): at the first rank below the floor, or one past the first whose
@@ -1993,7 +1996,7 @@ __device__ __noinline__ uint32_t deep_bins(const FinishArgs& a, const RowParams&
       if (topk && jl == kNone) {
         k_topp = kNone;
       } else {
-        if (jl != jh || jh == kNone) return undecided;
+        if (jl != jh || jh == kNone) return cut_open;
         k_topp = jh + 1;
       }
     }
@@ -2057,7 +2060,7 @@ __device__ __noinline__ uint32_t deep_bins(const FinishArgs& a, const RowParams&
   } else if (jp == jc) {
     pick_rank = jc;
   } else {
-    return undecided;
+    return draw_open;
   }
   uint32_t pi = kNone;
   for (uint32_t i = tid; i < P; i += kThreads)
