@@ -206,8 +206,9 @@ __global__ __launch_bounds__(kThreads) void matvec_kernel(const uint8_t* __restr
 // thread t + 8's (the second 32), moved by DPP. A quad past the row's end adds +0.0, which changes nothing
 // (a partial starts from +0.0 and is never -0.0).
 //
-// At 248,320 x 2,048, by events (us; a unit per lane before): Q6_K 127.7 to 89.8, 4.6 TB/s of weights and
-// about 4.7 VALU instructions per weight (62 us at full issue); Q5_K 111.7 to 71.5; Q4_K 110.7 to 61.7.
+// At 248,320 x 2,048, by events (us; a unit per lane before): Q6_K 127.7 to 86.8, 4.8 TB/s of weights and, by the
+// counters, 5.0 VALU instructions per weight (65 us at full issue); Q5_K 127.7 to 72.3, 5.2 per weight (68 us);
+// Q4_K 111.6 to 54.2, 3.8 per weight (49 us).
 constexpr uint32_t kQuadStride = 132;  // LDS floats per quad of x (see quad_kernel)
 typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x2_u __attribute__((ext_vector_type(2), aligned(2)));

@@ -55,7 +55,7 @@ constexpr uint32_t kArgLoads = 8;  // 16-byte loads in flight per thread
 // the row's `arrived`, and the slice that brings the count to `parts` reads the slices' bests
 // (device-coherent), writes the row and clears the count for the next call.
 // One workgroup's loads bound a lone row (1 MB at 10 GB/s with one 16-byte load per thread in flight):
-// a row of 248,320 values and embed_rows of its pick took 98.8 us, and take 11.4 as 61 slices of 4,096.
+// a row of 248,320 values and embed_rows of its pick took 98.8 us, and take 11.2 as 49 slices of 5,120.
 template <bool kVec>
 __global__ __launch_bounds__(kArgThreads) void argmax_kernel(const float* __restrict__ logits,
                                                              uint64_t row_stride, uint32_t n, uint32_t parts,
@@ -163,8 +163,9 @@ hipError_t accept(hipStream_t stream, const uint32_t* picks, const uint32_t* sta
   return hipGetLastError();
 }
 
-// Slices per row: enough workgroups for three per CU, of at least 4,096 values (greedy_kernel's length:
-// the same work per slice) and a multiple of 1,024, so that their 16-byte groups stay aligned. From
+// Slices per row: as many as make three workgroups per CU over the call's rows, of at least 4,096 values
+// (greedy_kernel's least) and, rounded up, of a multiple of 1,024, so that their 16-byte groups stay aligned:
+// at 248,320 values 49 of 5,120 for one row, 41 of 6,144 for 16, 3 of 82,944 for 256. From
 // kArgGroups rows on a row is one workgroup's, so n_rows * parts stays under 2 * kArgGroups wherever
 // the slices' bests are used. Without scratch (a captured call) every row is one workgroup's: a lone row of
 // 248,320 values 31.5 us in a replayed graph (97 with one load per thread in flight), against 4.8 in slices.
